@@ -81,10 +81,25 @@ def dispatcher_kernel_names():
     for ab in ("nn", "nt", "tn", "tt"):
         for tag in tiles:
             names.append(f"forge_gemm_batch_{ab}_{tag}")
-    # eight-wave 64x128 tile: plain NN, every epilogue kind, batched NN/NT/TN
+    # 64x128 tile of two groups: plain NN, fused epilogue, batched NN/NT/TN
     names.append("forge_gemm_nn_64x128x32_x8")
     names += [f"forge_gemm_{ab}_64x128x32_x8_e" for ab in ("nn", "nt", "tn", "tt")]
     names += [f"forge_gemm_batch_{ab}_64x128x32_x8" for ab in ("nn", "nt", "tn")]
+    # tiles whose groups of waves share K, and the direct tile: every kind
+    for tag in ("128x128x32_x8", "64x128x32_x8", "64x64x32_x16", "32x32x32_d"):
+        names.append(f"forge_gemm_nn_{tag}")
+        for ab in ("nn", "nt", "tn", "tt"):
+            names += [f"forge_gemm_{ab}_{tag}_{kind}" for kind in "esrk"]
+            names.append(f"forge_gemm_batch_{ab}_{tag}")
+    # guarded tiles: fused epilogue and plain NN; batched where products are
+    # split in K
+    guarded = ("128x128x32_2x2_g", "64x128x32_2x2_g", "64x64x16_2x2_g", "128x128x32_2x2_g8",
+               "64x128x32_2x2_g8", "64x64x32_2x2_g16", "64x64x32_2x2_gw", "32x32x32_2x2_gd")
+    for tag in guarded:
+        names.append(f"forge_gemm_nn_{tag}")
+        names += [f"forge_gemm_{ab}_{tag}_e" for ab in ("nn", "nt", "tn", "tt")]
+    for tag in ("64x64x32_2x2_g16", "32x32x32_2x2_gd"):
+        names += [f"forge_gemm_batch_{ab}_{tag}" for ab in ("nn", "nt", "tn", "tt")]
     names += ["forge_gemm_splitk_reduce_v", "forge_gemm_splitk_reduce_s"]
     for op in ("softmax", "layer_norm", "rms_norm", "softmax_bwd", "layer_norm_bwd", "rms_norm_bwd"):
         for v in (1, 2, 4, 8, 16):
@@ -110,7 +125,7 @@ def dispatcher_kernel_names():
               "forge_count_neq", "forge_count_final", "forge_count_neq_u32",
               "forge_count_final_u32", "forge_sgd_v", "forge_sgd_s", "forge_row_rms_parts",
               "forge_row_sq_parts"]
-    names += ["forge_fill_v", "forge_fill_s", "forge_fill_seq", "forge_causal_mask",
+    names += ["forge_copy_many", "forge_fill_v", "forge_fill_s", "forge_fill_seq", "forge_causal_mask",
               "forge_sum_cols_v", "forge_sum_cols_s", "forge_sum_cols_final", "forge_sum_cols_final2",
               "forge_sum_cols_final_v", "forge_sum_cols_final2_v",
               "forge_sum_cols_p4", "forge_sum_cols_p8", "forge_sum_cols_p16",
