@@ -82,6 +82,42 @@ def test_values_that_are_not_finite(rt, tile):
     assert np.all(np.abs(C[ok] - ref[ok]) <= (K + 8) * U32 * scale[ok])
 
 
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("K", [96, 544])
+def test_values_whose_parts_are_not_f32(rt, tile, ta, tb, K):
+    """Values whose bf16 parts behave otherwise than they do in f32: infinities
+    against the smallest values (both ways round), a NaN with its payload in
+    the low bits only, a product beyond the f32 range against a sum of the
+    other sign, and the largest finite value against zeros and ones.  Each
+    output is what f32 multiply-adds give: NaN and infinities as the f64
+    product's, the others within (K + 8) u of |A| |B|."""
+    M, N = (int(x) for x in tile.split("x")[:2])
+    say(f"parts that are not f32: {tile} ta={ta} tb={tb} K={K}")
+    A, B = synth.uniform((M, K), 11), synth.uniform((K, N), 12)
+    big = np.finfo(np.float32).max
+    B[5, :] = np.where(np.arange(N) % 2, 2.0 ** -140, -2.0 ** -149)
+    A[1, 5], A[2, 5] = np.inf, -np.inf
+    A[3, 20], B[20, 3] = 2.0 ** -149, np.inf
+    A[4, 20], B[K - 1, 4] = -2.0 ** -135, -np.inf
+    A[5, 9] = np.array([0x7F800001], np.uint32).view(np.float32)[0]
+    A[6, :], A[6, 0], A[6, 1] = 0.0, -3e38, 2e19
+    B[0, :], B[1, :] = 1.0, 2e19
+    A[7, :], A[7, 0] = 0.0, big
+    a, b = (A.T.copy() if ta else A), (B.T.copy() if tb else B)
+    C = product(rt, a, b, M, N, K, ta, tb, tile)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+    assert np.array_equal(np.isnan(C), np.isnan(ref)), np.argwhere(np.isnan(C) != np.isnan(ref))[:4]
+    inf = np.isinf(ref)
+    assert np.array_equal(np.isinf(C), inf), np.argwhere(np.isinf(C) != inf)[:4]
+    assert np.array_equal(C[inf], ref[inf].astype(np.float32))
+    ok = np.isfinite(ref)
+    scale = np.abs(np.where(np.isfinite(A), A, 0)).astype(np.float64) @ \
+        np.abs(np.where(np.isfinite(B), B, 0)).astype(np.float64)
+    assert np.all(np.abs(C[ok] - ref[ok]) <= (K + 8) * U32 * scale[ok])
+
+
 @pytest.mark.parametrize("exponent", [-126, -118, -110, -100, -60, 60, 100, 118])
 def test_range_of_the_parts(rt, exponent):
     """Operands scaled by 2^exponent against operands of order one: within
