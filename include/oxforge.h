@@ -210,10 +210,15 @@ forge_status forge_fill(forge_runtime *rt, forge_stream *stream,
  * gemm.rs:202-373): C[M,N] = A[M,K] * B[K,N], row-major, C overwritten.
  * f32 operands and results, not the reference's TF32: each operand value is
  * split exactly into three bf16 parts and the product formed from six bf16
- * matrix instructions with f32 accumulation (v_mfma_f32_16x16x32_bf16),
- * with a smaller error against 64 bits than the f32 matrix instructions
- * give; infinities and NaN propagate as in f32 (operand values under 2^-109
- * keep an absolute error of 2^-134).  Any M, N, K >= 0 (the reference
+ * matrix instructions with f32 accumulation (v_mfma_f32_16x16x32_bf16).  What
+ * is left out of a product is at most 2^-24 (1 + 2^-10) of it, and the error
+ * against 64 bits is smaller than that of f32 multiply-adds in sums of four
+ * products or more (2-norm, uniform(-1, 1): K = 4 2.6e-8 against 4.0e-8,
+ * K = 1024 8.2e-8 against 5.8e-7; a longer sum with a single product that is
+ * not zero is off by up to two roundings of it).  Sums of up to three
+ * products, sums that are not finite, and the rows and columns of values that
+ * are not whole multiples of 2^-133 are formed by the f32 matrix instructions
+ * (v_mfma_f32_16x16x4_f32).  Any M, N, K >= 0 (the reference
  * asserts multiples of 16).  Outputs whose tiles leave three quarters of the
  * CUs idle, with K >= 2048, are computed as K slices summed in slice order
  * (deterministic; tile, sum order and slices depend only on M, N and K, the

@@ -39,7 +39,8 @@ def test_group_and_guard_edges(rt, tile, ta, tb):
     """K from one slab to every count of slabs per group (with a ragged last
     slab on guarded tiles), one row or column short of the tile and one past
     it: within (K + 8) u of |A| |B| of the f64 product (every order of K
-    rounded additions; the parts left out of a product are below u of it)."""
+    rounded additions; the parts left out of a product are at most
+    (1 + 2^-10) u of it)."""
     bm, bn = (int(x) for x in tile.split("x")[:2])
     guarded = "_g" in tile
     sizes = [(bm, bn)] + ([(bm - 1, bn + 1), (1, 3), (bm + 3, bn - 2)] if guarded else [])
@@ -116,6 +117,80 @@ def test_values_whose_parts_are_not_f32(rt, tile, ta, tb, K):
     scale = np.abs(np.where(np.isfinite(A), A, 0)).astype(np.float64) @ \
         np.abs(np.where(np.isfinite(B), B, 0)).astype(np.float64)
     assert np.all(np.abs(C[ok] - ref[ok]) <= (K + 8) * U32 * scale[ok])
+
+
+# Mantissas whose parts leave out the most: of a truncated hi, of a rounded one.
+WORST = np.array([0x3F80FF80, 0x3F807F80, 0x3F817F80, 0x3FFFFF80, 0x3F80807F, 0xBF80FF80],
+                 np.uint32).view(np.float32)
+
+
+@pytest.mark.parametrize("tile", [t for t in TILES if "_g" in t] + [None])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_short_sums(rt, tile, ta, tb):
+    """Sums of up to three products are formed by f32 multiply-adds, K u of
+    |A| |B|, one product rounded once; sums of four keep within that bound and
+    what the parts leave out.  Among the operands are the mantissas of which
+    that is the most."""
+    M, N = (int(x) + 1 for x in tile.split("x")[:2]) if tile else (70, 300)
+    rng = np.random.default_rng(13)
+    for K in (1, 2, 3, 4):
+        say(f"short sums {tile} ta={ta} tb={tb} K={K}")
+        for worst in (False, True):
+            A = rng.choice(WORST, (M, K)) if worst else synth.uniform((M, K), K)
+            B = rng.choice(WORST, (K, N)) if worst else synth.uniform((K, N), K + 20)
+            C = product(rt, A.T.copy() if ta else A, B.T.copy() if tb else B, M, N, K, ta, tb, tile)
+            a, b = A.astype(np.float64), B.astype(np.float64)
+            tol = (K * (1 + K * U32) if K < 4 else K + 1) * U32 * (np.abs(a) @ np.abs(b))
+            assert K > 1 or np.array_equal(C, A * B)
+            assert np.all(np.abs(C - a @ b) <= tol), (K, worst)
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_sums_of_one_product(rt, tile):
+    """One product that is not zero in each sum: what the parts leave out,
+    (1 + 2^-10) u of it, and two roundings (of the small parts' sum, below
+    2^-7 of it, and of the result)."""
+    M, N = (int(x) for x in tile.split("x")[:2])
+    rng = np.random.default_rng(14)
+    for K in (32, 288):
+        say(f"sums of one product {tile} K={K}")
+        A, B = np.zeros((M, K), np.float32), rng.choice(WORST, (K, N))
+        A[np.arange(M), rng.integers(0, K, M)] = rng.choice(WORST, M)
+        C = product(rt, A, B, M, N, K, tile=tile)
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+        assert np.all(np.abs(C - ref) <= (2 + 2.0 ** -6) * U32 * np.abs(ref)), K
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_smallest_operands(rt, tile, ta, tb):
+    """Rows of A and columns of B down to the smallest f32 values, whose parts
+    bf16 does not hold, against values of 2^100: within (K + 8) u of |A| |B|
+    like any others, and the elements of other rows and columns are bit for
+    bit those of a product without them."""
+    M, N = (int(x) for x in tile.split("x")[:2])
+    for K in (96, 544):
+        say(f"smallest operands {tile} ta={ta} tb={tb} K={K}")
+        A, B = synth.uniform((M, K), 15), synth.uniform((K, N), 16)
+        A[:, ::7] *= np.float32(2.0 ** 100)
+        B[3::7, :] *= np.float32(2.0 ** 100)
+        flat = lambda X, t: X.T.copy() if t else X  # noqa: E731
+        plain = product(rt, flat(A, ta), flat(B, tb), M, N, K, ta, tb, tile)
+        rows, cols = {}, {}
+        for i, e in enumerate((-149, -148, -140, -134, -133, -126, -118, -111)):
+            r, c = (3 * i + 1) % M, (3 * i + 2) % N
+            A[r] = np.ldexp(synth.uniform((K,), 30 + i), e).astype(np.float32)
+            rows[r] = e
+            if i % 2:
+                B[:, c] = np.ldexp(synth.uniform((K,), 40 + i), e).astype(np.float32)
+                cols[c] = e
+        C = product(rt, flat(A, ta), flat(B, tb), M, N, K, ta, tb, tile)
+        a, b = A.astype(np.float64), B.astype(np.float64)
+        err, scale = np.abs(C - a @ b), np.abs(a) @ np.abs(b)
+        # (f32 results under 2^-126 are whole multiples of 2^-149)
+        assert np.all(err <= (K + 8) * U32 * scale + K * 2.0 ** -149), float((err / scale).max())
+        other = np.ix_([r for r in range(M) if r not in rows], [c for c in range(N) if c not in cols])
+        assert np.array_equal(C[other], plain[other])
 
 
 @pytest.mark.parametrize("exponent", [-126, -118, -110, -100, -60, 60, 100, 118])
