@@ -216,9 +216,9 @@ forge_status forge_fill(forge_runtime *rt, forge_stream *stream,
  * products or more (2-norm, uniform(-1, 1): K = 4 2.6e-8 against 4.0e-8,
  * K = 1024 8.2e-8 against 5.8e-7; a longer sum with a single product that is
  * not zero is off by up to two roundings of it).  Sums of up to three
- * products, sums that are not finite, and the rows and columns of values that
- * are not whole multiples of 2^-133 are formed by the f32 matrix instructions
- * (v_mfma_f32_16x16x4_f32).  Any M, N, K >= 0 (the reference
+ * products, sums that are not finite, and sums to which what bf16's smallest
+ * value cuts off operands under 2^-110 could matter are formed by the f32
+ * matrix instructions (v_mfma_f32_16x16x4_f32).  Any M, N, K >= 0 (the reference
  * asserts multiples of 16).  Outputs whose tiles leave three quarters of the
  * CUs idle, with K >= 2048, are computed as K slices summed in slice order
  * (deterministic; tile, sum order and slices depend only on M, N and K, the

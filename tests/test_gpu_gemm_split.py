@@ -193,6 +193,45 @@ def test_smallest_operands(rt, tile, ta, tb):
         assert np.array_equal(C[other], plain[other])
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("tiles", [("128x128x32_x", "64x128x32_x", "64x64x32_x", "128x128x32_2x2_g",
+                                    "64x128x32_2x2_g", "64x64x16_2x2_g", "64x64x32_2x2_gw"),
+                                   ("128x128x32_x8", "64x128x32_x8", "128x128x32_2x2_g8",
+                                    "64x128x32_2x2_g8"),
+                                   ("64x64x32_x16", "64x64x32_2x2_g16"),
+                                   ("32x32x32_d", "32x32x32_2x2_gd")])
+def test_elements_do_not_depend_on_the_tile(rt, tiles, ta, tb):
+    """Operands with every kind of value that the parts do not carry, in some
+    rows and columns, among others, and as the small values of otherwise
+    ordinary rows (as activations have): tiles of the same number of groups
+    give the same bits, whichever elements share a tile."""
+    M, N, K = 128, 128, 544
+    say(f"elements alone {tiles[0]} ta={ta} tb={tb}")
+    rng = np.random.default_rng(17)
+    A, B = synth.uniform((M, K), 18), synth.uniform((K, N), 19)
+    A[rng.random((M, K)) < 0.02] = 1e-40           # irrelevant to most sums
+    A[3], A[70] = np.ldexp(A[3], -120), np.ldexp(A[70], -140)
+    A[5], A[6, ::2] = 0.0, 1e-39
+    A[5, 9] = 1e-41
+    B[:, 33] = np.ldexp(B[:, 33], -130)
+    B[::3, 90] = 0.0
+    B[9, 90] = 2.0 ** 100
+    A[40, 17], A[41, 18], A[42, 19] = np.inf, np.nan, -np.inf
+    B[17, 4], B[18, 5], B[100, 6] = 1e-42, 0.0, 3e38
+    A[43, 100] = 3e38
+    a, b = (A.T.copy() if ta else A), (B.T.copy() if tb else B)
+    C = [product(rt, a, b, M, N, K, ta, tb, tile) for tile in tiles]
+    for tile, c in zip(tiles, C):
+        assert np.array_equal(c.view(np.uint32)[np.isfinite(c)],
+                              C[0].view(np.uint32)[np.isfinite(c)]), tile
+        assert np.array_equal(c, C[0], equal_nan=True), tile
+    with np.errstate(invalid="ignore", over="ignore"):
+        a64, b64 = A.astype(np.float64), B.astype(np.float64)
+        ref, scale = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    ok = np.isfinite(scale) & (scale < 1e38)
+    assert np.all(np.abs(C[0][ok] - ref[ok]) <= (K + 8) * U32 * scale[ok] + K * 2.0 ** -149)
+
+
 @pytest.mark.parametrize("exponent", [-126, -118, -110, -100, -60, 60, 100, 118])
 def test_range_of_the_parts(rt, exponent):
     """Operands scaled by 2^exponent against operands of order one: within
