@@ -916,7 +916,7 @@ int choose_splits(forge_runtime* rt, size_t M, size_t N, size_t K, GemmReads rea
 }
 
 constexpr long long kUnguardedMaxPitch = 1LL << 21;
-constexpr long long kGuardedMaxPitch = 1LL << 23;
+constexpr long long kGuardedMaxPitch = 1LL << 23;  // X_GUARDED_MAX_PITCH of gemm_x.hpp
 
 // Validates one product and fills its kernel arguments; *reads reports how
 // its operands can be read.
@@ -1011,7 +1011,7 @@ forge_status gemm_split_launch(forge_runtime* rt, forge_stream* s, int ta, int t
                                const GemmArgs& a, const GemmConfig& cfg, int splits,
                                float* ws) {
     const size_t mn = (size_t)a.M * (size_t)a.N;
-    const int slabs = (a.K + cfg.bk - 1) / cfg.bk;
+    const int slabs = (int)(((size_t)a.K + cfg.bk - 1) / cfg.bk);
     const int ks = (slabs + splits - 1) / splits * cfg.bk;
     GemmBatchArgs b{};
     b.count = splits;

@@ -267,6 +267,43 @@ def test_pitch_beyond_32_bit_offsets(rt, ta, tb, M, N, K):
         assert np.all(np.abs(C[r] - row @ b) <= (K + 8) * U32 * (np.abs(row) @ np.abs(b))), r
 
 
+@pytest.mark.parametrize("tb,tile", [(0, "128x128x32_2x2_g"), (0, "128x128x32_2x2_g8"),
+                                     (1, "128x128x32_2x2_g"), (1, "64x128x32_2x2_g8"), (0, None)])
+def test_pitch_up_to_32_bit_offsets(rt, tb, tile):
+    """k contiguous at a pitch just under 2^23 floats, whose 128 rows reach
+    byte offsets beyond 2^31 from a slab's first value: zeros but for some k
+    near the ends and the middle, in rows on either side of that."""
+    K = 2**23 - 3
+    M, N = (3, 128) if tb else (128, 3)
+    say(f"pitch {K} tb={tb} {tile}")
+    R, S = (N, M) if tb else (M, N)  # rows of that pitch, and of the other operand
+    ks = np.r_[0:9, K // 2:K // 2 + 9, K - 9:K]
+    big, small = synth.uniform((R, len(ks)), 21), synth.uniform((len(ks), S), 22)
+    dbig, dsmall = rt.empty((R, K)), rt.empty((M, K) if tb else (K, N))
+    for d in (dbig, dsmall):
+        rt.fill(d, 0.0)
+    for i in range(0, len(ks), 9):
+        for r in range(R):
+            dbig.view(r * K + int(ks[i]), (9,)).upload(np.ascontiguousarray(big[r, i:i + 9]))
+        if tb:
+            for m in range(M):
+                dsmall.view(m * K + int(ks[i]), (9,)).upload(
+                    np.ascontiguousarray(small[i:i + 9, m]))
+        else:
+            dsmall.view(int(ks[i]) * N, (9, N)).upload(np.ascontiguousarray(small[i:i + 9]))
+    A, B = (dsmall, dbig) if tb else (dbig, dsmall)
+    dC = rt.empty((M, N))
+    if tile:
+        rt.gemm_ex_tile(tile, A, B, dC, M, N, K, trans_b=tb)
+    else:
+        rt.gemm_ex(A, B, dC, M, N, K, trans_b=tb)
+    C = dC.numpy().T if tb else dC.numpy()
+    a, b = big.astype(np.float64), small.astype(np.float64)
+    assert np.all(np.abs(C - a @ b) <= (len(ks) + 8) * U32 * (np.abs(a) @ np.abs(b)))
+    for d in (dbig, dsmall, dC):
+        d.recycle()
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(64, 64, 2048), (1, 70, 2049), (33, 130, 2177), (16, 192, 4095),
                                    (65, 64, 3072)])
