@@ -873,6 +873,12 @@ const GemmConfig* instance_of(const GemmConfig& g, size_t M, size_t N, size_t K,
                : g.guarded;
 }
 
+// The instance of a named guarded tile for pitches beyond its 32-bit offsets:
+// the 64 x 64 tile of one group has one with 64-bit addresses (null: none).
+const GemmConfig* wide_instance(const GemmConfig* g) {
+    return g == &kGuard64x64 || g == &kGuardWide ? &kGuardWide : nullptr;
+}
+
 // The kernel for a product.
 const GemmConfig& choose_gemm(forge_runtime* rt, size_t M, size_t N, size_t K, GemmReads reads,
                               size_t count = 1) {
@@ -1541,8 +1547,8 @@ extern "C" forge_status forge_gemm_f32_tile(forge_runtime* rt, forge_stream* s,
                      (long long)K > kUnguardedMaxPitch || (long long)N > kUnguardedMaxPitch))
         return fail(FORGE_EINVAL, "shape %zux%zux%zu does not fit unguarded tile %s", M, N, K,
                     tile_tag);
-    if ((long long)std::max(K, N) > kGuardedMaxPitch && cfg != &kGuardWide)
-        return fail(FORGE_EINVAL, "row pitch is beyond tile %s", tile_tag);
+    if ((long long)std::max(K, N) > kGuardedMaxPitch) cfg = wide_instance(cfg);
+    if (!cfg) return fail(FORGE_EINVAL, "row pitch is beyond tile %s", tile_tag);
     if (M == 0 || N == 0) return FORGE_OK;
     GemmArgs a{};
     a.A = A.ptr;
@@ -1601,8 +1607,8 @@ extern "C" forge_status forge_gemm_ex_f32_tile(forge_runtime* rt, forge_stream* 
     GemmArgs a{};
     GemmReads reads = GemmReads::Guarded;
     FORGE_TRY(gemm_args(trans_a, trans_b, A, B, C, M, N, K, ep, &a, &reads));
-    if (reads == GemmReads::Wide && cfg != &kGuardWide)
-        return fail(FORGE_EINVAL, "row pitch is beyond tile %s", tile_tag);
+    if (reads == GemmReads::Wide) cfg = wide_instance(cfg);
+    if (!cfg) return fail(FORGE_EINVAL, "row pitch is beyond tile %s", tile_tag);
     if (!is_guarded(*cfg) &&
         (reads != GemmReads::Aligned || M % cfg->bm || N % cfg->bn || K % (size_t)cfg->bk))
         return fail(FORGE_EINVAL, "shape %zux%zux%zu does not fit unguarded tile %s", M, N, K,

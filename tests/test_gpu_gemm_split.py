@@ -267,6 +267,21 @@ def test_pitch_beyond_32_bit_offsets(rt, ta, tb, M, N, K):
         assert np.all(np.abs(C[r] - row @ b) <= (K + 8) * U32 * (np.abs(row) @ np.abs(b))), r
 
 
+def test_named_guarded_tile_takes_any_pitch(rt):
+    """The guarded 64 x 64 tile by name at a pitch above 2^23 floats, as the
+    plain and the fused product: what the dispatcher gives there."""
+    M, N, K = 2, 3, 2**23 + 5
+    say(f"named tile at pitch {K}")
+    A, B = rt.array(synth.uniform((M, K), 23)), rt.array(synth.uniform((K, N), 24))
+    ref, C, E = (rt.empty((M, N)) for _ in range(3))
+    rt.gemm(A, B, ref, M, N, K)
+    rt.gemm_tile("64x64x16_2x2_g", A, B, C, M, N, K)
+    rt.gemm_ex_tile("64x64x16_2x2_g", A, B, E, M, N, K)
+    assert np.array_equal(C.numpy(), ref.numpy()) and np.array_equal(E.numpy(), ref.numpy())
+    with pytest.raises(oxforge.ForgeError):
+        rt.gemm_tile("128x128x32_2x2_g", A, B, C, M, N, K)
+
+
 @pytest.mark.parametrize("tb,tile", [(0, "128x128x32_2x2_g"), (0, "128x128x32_2x2_g8"),
                                      (1, "128x128x32_2x2_g"), (1, "64x128x32_2x2_g8"), (0, None)])
 def test_pitch_up_to_32_bit_offsets(rt, tb, tile):
