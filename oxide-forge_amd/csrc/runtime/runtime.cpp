@@ -799,9 +799,11 @@ forge_status occupancy_cap_shmem(forge_runtime* rt, const char* name, int cap, s
     return FORGE_OK;
 }
 
-// Factor i of the comma-separated list in $OXFORGE_GEMM_EFF (a tuning knob: a
-// larger factor makes tile i of kChoice more likely), 1 without it.
-double tile_factor(int i) {
+// Tile g's factor from the comma-separated list in $OXFORGE_GEMM_EFF (a tuning
+// knob: a larger factor makes a tile more likely), 1 without one.  The list
+// keeps the order it has always had, also for tiles that are no longer
+// chosen, with later tiles after them.
+double tile_factor(const GemmConfig& g) {
     static const std::vector<double> env = [] {
         std::vector<double> v;
         if (const char* e = getenv("OXFORGE_GEMM_EFF")) {
@@ -813,7 +815,12 @@ double tile_factor(int i) {
         }
         return v;
     }();
-    return (size_t)i < env.size() && env[(size_t)i] > 0.0 ? env[(size_t)i] : 1.0;
+    static const GemmConfig* const order[] = {
+        &kTile128x256, &kTile128x128,   &kTile128x64,    &kTile64x128,  &kTile64x64,
+        &kTile64x128k2, &kTile128x128k2, &kTile64x64k4,  &kTile32x32};
+    for (size_t i = 0; i < env.size() && i < sizeof order / sizeof order[0]; i++)
+        if (order[i] == &g && env[i] > 0.0) return env[i];
+    return 1.0;
 }
 
 // Modelled time of count products of one shape on tile c, K in `slabs` slabs.
@@ -849,7 +856,7 @@ const TileTimes& choose_shape(forge_runtime* rt, size_t M, size_t N, size_t K, s
     for (int i = 0; i < kChoiceCount; i++) {
         const GemmConfig& g = *kChoice[i].cfg;
         if ((kg && g.kg != kg) || (g.kg > 1 && !g.direct() && slabs < 4)) continue;
-        double time = tile_time(kChoice[i], cus, M, N, count, slabs) / tile_factor(i);
+        double time = tile_time(kChoice[i], cus, M, N, count, slabs) / tile_factor(g);
         if (M % g.bm || N % g.bn || K % 32) time *= kChoice[i].edge;
         if (!best || time < best_time) {
             best = &kChoice[i];

@@ -1,6 +1,10 @@
 """The products' bf16 parts (gemm_x.hpp): the range of values they hold, the
 values that are not finite, and the edges of the tiles that split K over
 groups of waves."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -265,6 +269,25 @@ def test_pitch_beyond_32_bit_offsets(rt, ta, tb, M, N, K):
     for r in sorted({0, 1, M // 2, M - 1}):
         row = a[r].astype(np.float64)
         assert np.all(np.abs(C[r] - row @ b) <= (K + 8) * U32 * (np.abs(row) @ np.abs(b))), r
+
+
+@pytest.mark.parametrize("factors,tile", [("1,50", "128x128x32_x_e"), ("1,1,50,50", "64x128x32_x_e"),
+                                          ("1,1,1,1,1,50", "64x128x32_x8_e"),
+                                          ("1,1,1,1,1,1,1,50", "64x64x32_x16_e"),
+                                          ("1,1,1,1,1,1,1,1,50", "32x32x32_d_e")])
+def test_order_of_the_tile_factors(factors, tile):
+    """OXFORGE_GEMM_EFF (read once by a process) keeps its documented order:
+    128x256, 128x128, 128x64, 64x128, 64x64 and the 64x128 tile of two groups,
+    then the later ones."""
+    say(f"tile factors {factors}")
+    code = ("import oxforge\nwith oxforge.Runtime(0) as rt:\n"
+            "    print(rt.gemm_kernel_name(1024, 1024, 1024, fused=True))")
+    env = dict(os.environ, OXFORGE_GEMM_EFF=factors,
+               PYTHONPATH=os.path.dirname(os.path.dirname(oxforge.__file__)))
+    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True,
+                         timeout=60)
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.strip().endswith(tile)
 
 
 def test_named_guarded_tile_takes_any_pitch(rt):
