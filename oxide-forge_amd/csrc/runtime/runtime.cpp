@@ -699,18 +699,19 @@ struct GemmConfig {
     const char* tag;  // e.g. "128x128x32_x"
     int bm, bn, bk, kg;
     const GemmConfig* guarded;
+    bool is_guarded = false;
     bool direct() const { return bm == 32; }  // a group is one wave, not four
     int threads() const { return (direct() ? 64 : 256) * kg; }
 };
 
-const GemmConfig kGuard128x128 = {"128x128x32_2x2_g", 128, 128, 32, 1, nullptr};
-const GemmConfig kGuard128x128k2 = {"128x128x32_2x2_g8", 128, 128, 32, 2, nullptr};
-const GemmConfig kGuard64x128k2 = {"64x128x32_2x2_g8", 64, 128, 32, 2, nullptr};
-const GemmConfig kGuard64x64k4 = {"64x64x32_2x2_g16", 64, 64, 32, 4, nullptr};
-const GemmConfig kGuard64x128 = {"64x128x32_2x2_g", 64, 128, 32, 1, nullptr};
-const GemmConfig kGuard64x64 = {"64x64x16_2x2_g", 64, 64, 32, 1, nullptr};
-const GemmConfig kGuardWide = {"64x64x32_2x2_gw", 64, 64, 32, 1, nullptr};
-const GemmConfig kGuard32x32 = {"32x32x32_2x2_gd", 32, 32, 32, 8, nullptr};
+const GemmConfig kGuard128x128 = {"128x128x32_2x2_g", 128, 128, 32, 1, nullptr, true};
+const GemmConfig kGuard128x128k2 = {"128x128x32_2x2_g8", 128, 128, 32, 2, nullptr, true};
+const GemmConfig kGuard64x128k2 = {"64x128x32_2x2_g8", 64, 128, 32, 2, nullptr, true};
+const GemmConfig kGuard64x64k4 = {"64x64x32_2x2_g16", 64, 64, 32, 4, nullptr, true};
+const GemmConfig kGuard64x128 = {"64x128x32_2x2_g", 64, 128, 32, 1, nullptr, true};
+const GemmConfig kGuard64x64 = {"64x64x16_2x2_g", 64, 64, 32, 1, nullptr, true};
+const GemmConfig kGuardWide = {"64x64x32_2x2_gw", 64, 64, 32, 1, nullptr, true};
+const GemmConfig kGuard32x32 = {"32x32x32_2x2_gd", 32, 32, 32, 8, nullptr, true};
 const GemmConfig kTile128x256 = {"128x256x32_x", 128, 256, 32, 1, nullptr};
 const GemmConfig kTile128x128 = {"128x128x32_x", 128, 128, 32, 1, &kGuard128x128};
 const GemmConfig kTile128x64 = {"128x64x32_x", 128, 64, 32, 1, nullptr};
@@ -735,7 +736,7 @@ const GemmConfig* tile_by_tag(const char* tag) {
     return nullptr;
 }
 
-bool is_guarded(const GemmConfig& g) { return strstr(g.tag, "_g") != nullptr; }
+bool is_guarded(const GemmConfig& g) { return g.is_guarded; }
 
 // The tiles the dispatcher chooses from and the time model of the choice
 // (choose_shape), in microseconds: what a CU takes per K slab with one
