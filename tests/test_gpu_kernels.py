@@ -1044,7 +1044,9 @@ def test_gemm_split_k_vs_oracle(rt, tile, splits, M, N, K):
 
 
 TILES = ["128x128x32_x", "128x64x32_x", "64x128x32_x", "64x64x32_x", "64x128x32_x8",
-         "64x64x16_2x2_g"]
+         "64x64x16_2x2_g", "128x128x32_x8", "64x64x32_x16", "32x32x32_d", "128x128x32_2x2_g",
+         "64x128x32_2x2_g", "128x128x32_2x2_g8", "64x128x32_2x2_g8", "64x64x32_2x2_g16",
+         "64x64x32_2x2_gw", "32x32x32_2x2_gd"]
 
 
 @pytest.mark.parametrize("tile", TILES)
@@ -1234,7 +1236,8 @@ def test_gemm_epilogue_row_statistics_and_column_sums(rt, tile, ta, tb, N):
     the GEMM bar (1e-4 of the f64 result on the GPU's own Y1); sums within
     their rounding bounds; the parameter step bit for bit against the
     returned sums.  N = 192 gives 6 partials per row (the unguarded tiles'
-    scalar row-scale loads), N = 352 shapes no unguarded tile divides."""
+    scalar row-scale loads), N = 352 shapes no unguarded tile but the direct
+    one divides."""
     M, K = 256, 160
     bn = 64 if tile is None else int(tile.split("x")[1])
     if tile is not None and N % bn:
@@ -1308,6 +1311,39 @@ def test_gemm_epilogue_statistics_on_split_and_guarded_products(rt):
     assert np.all(cs.numpy() == 0) and np.all(par.numpy() == 2.0)
     with pytest.raises(oxforge.ForgeError):  # row_div without row statistics
         rt.gemm_ex(dA, dB, dY1, 64, 128, 4096, row_div=1)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,tag", [(1152, 256, 128, "64x64x32_x16"),
+                                       (768, 1536, 192, "64x128x32_x8"),
+                                       (2048, 2048, 256, "128x128x32_x8"),
+                                       (256, 256, 128, "32x32x32_d")])
+def test_gemm_batch_and_sum_on_tiles_that_share_k(rt, M, N, K, tag, ta, tb):
+    """Shapes whose single product takes a tile of several groups: a batch of
+    two, which takes a tile of as many groups, and a sum of two products of
+    half the depth equal forge_gemm_ex_f32 bit for bit."""
+    name = rt.gemm_kernel_name(M, N, K, bool(ta), bool(tb), True)
+    say(f"gemm batch and sum {M}x{N}x{K} ta={ta} tb={tb}: {name}")
+    assert name.endswith(tag + "_e")
+    As = [synth.uniform((K, M) if ta else (M, K), 95 + z) for z in range(2)]
+    Bs = [synth.uniform((N, K) if tb else (K, N), 97 + z) for z in range(2)]
+    bias = rt.array(synth.uniform((N,), 99))
+    dA, dB = [rt.array(a) for a in As], [rt.array(b) for b in Bs]
+    C = [rt.empty((M, N)) for _ in range(4)]
+    rt.gemm_batch([(dA[z], dB[z], C[z], dict(bias=bias)) for z in range(2)], M, N, K,
+                  trans_a=ta, trans_b=tb)
+    for z in range(2):
+        rt.gemm_ex(dA[z], dB[z], C[2], M, N, K, trans_a=ta, trans_b=tb, bias=bias)
+        assert np.array_equal(C[z].numpy(), C[2].numpy())
+    half = K // 2
+    cut = lambda X, t, z: np.ascontiguousarray(  # noqa: E731
+        X[z * half:(z + 1) * half] if t else X[:, z * half:(z + 1) * half])
+    rt.gemm_sum([rt.array(cut(As[1], ta, z)) for z in range(2)],
+                [rt.array(cut(Bs[1], not tb, z)) for z in range(2)], C[3], M, N, half,
+                trans_a=ta, trans_b=tb, bias=bias)
+    assert np.array_equal(C[3].numpy(), C[2].numpy())
+    ref = orc.gemm_f64(As[1], Bs[1], ta, tb) + bias.numpy()
+    assert np.max(np.abs(C[2].numpy() - ref)) / np.max(np.abs(ref)) <= 1e-4
 
 
 @pytest.mark.parametrize("M,N,K,ta,tb,fused", [(4096, 4096, 4096, 0, 0, 0),
@@ -1586,8 +1622,8 @@ def test_operands_beyond_4gib(rt):
 
 def test_gemm_pitch_beyond_unguarded_limit(rt):
     """A row pitch above 2^21 floats (A^T of [64, 2^21 + 64] in a TN
-    product) goes to the bounds-guarded kernel, whose offsets are 64-bit;
-    rows on both sides of the 2^21 boundary match the f64 oracle."""
+    product) goes to the bounds-guarded kernel (32-bit offsets from each
+    slab's first element, to pitches of 2^23); rows on both sides of the 2^21 boundary match the f64 oracle."""
     M, N, K = 2**21 + 64, 64, 64
     say(f"gemm pitch {M} (tn)")
     assert "_g" in rt.gemm_kernel_name(M, N, K, trans_a=True, fused=True)
