@@ -2,7 +2,8 @@
 """Benchmark of the MI355X-native OxideForge compute core (one GPU).
 
 Headline (BASELINE.json metric, configs[2]): f32 GEMM C = A * B at
-M = N = K = 4096, TFLOP/s, with its fraction of the fp32-MFMA peak.  A "step"
+M = N = K = 4096, TFLOP/s, with its fraction of the rate that six bf16 matrix
+instructions per product allow.  A "step"
 is one GEMM launch over inputs already resident in HBM; the timed region is
 bracketed by synchronisation and timed with HIP events on the stream the
 kernel runs on, and every figure is the median over five groups of
@@ -38,7 +39,9 @@ sys.path.insert(0, ROOT)
 from oxforge import synth  # noqa: E402  (seeded inputs; the package, not the oracle)
 
 METRIC = "f32 GEMM TFLOP/s (% fp32-MFMA peak); transformer layer tokens/sec, 1 GPU"
-PEAK_FP32_MFMA_TFLOPS = 157.3
+# f32 products run as six bf16 matrix instructions each; those reach 2146
+# TFLOP/s in a register-only loop, so 358 of f32 products.
+PEAK_GEMM_TFLOPS = 358.0
 PEAK_HBM_GBS = 8000.0
 
 
@@ -135,7 +138,7 @@ def secondary(rt, steps, warmup, extended):
     log("gemm 8192x1024x4096")
     t, ms = gemm_tflops(rt, 8192, 1024, 4096, steps, warmup)
     out["gemm_8192x1024x4096"] = {"tflops": round(t, 2), "ms": round(ms, 4),
-                                  "frac_mfma_peak": round(t / PEAK_FP32_MFMA_TFLOPS, 4)}
+                                  "frac_mfma_peak": round(t / PEAK_GEMM_TFLOPS, 4)}
 
     log("transpose 8192x4096")
     R, C = 8192, 4096
@@ -294,7 +297,7 @@ def transformers(rt, steps, warmup):
     out["transformer_c4_inference"] = {
         "tokens_per_s": round(S / (ms * 1e-3), 1), "ms_per_forward": round(ms, 4),
         "tflops": round(flops / (ms * 1e-3) / 1e12, 2),
-        "frac_mfma_peak": round(flops / (ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4)}
+        "frac_mfma_peak": round(flops / (ms * 1e-3) / 1e12 / PEAK_GEMM_TFLOPS, 4)}
     T.close()
     X.recycle()
     Y.recycle()
@@ -318,7 +321,7 @@ def transformers(rt, steps, warmup):
     out["transformer_c5_training"] = {
         "tokens_per_s": round(S / (ms * 1e-3), 1), "ms_per_step": round(ms, 3),
         "tflops_algorithmic": round(flops / (ms * 1e-3) / 1e12, 2),
-        "frac_mfma_peak": round(flops / (ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4)}
+        "frac_mfma_peak": round(flops / (ms * 1e-3) / 1e12 / PEAK_GEMM_TFLOPS, 4)}
     T.close()
     for d in (X, dY, Y, dX):
         d.recycle()
@@ -749,8 +752,8 @@ def main() -> int:
         "config": {"workload": "f32 GEMM C=A*B, M=N=K=4096, row-major (BASELINE configs[2])",
                    "kernel": kernel, "device": props.get("arch")},
         "roofline": {"bound": "mfma", "achieved": round(tflops, 3),
-                     "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(tflops / PEAK_FP32_MFMA_TFLOPS, 4), "traffic": traffic},
+                     "peak": PEAK_GEMM_TFLOPS, "unit": "TFLOP/s",
+                     "frac": round(tflops / PEAK_GEMM_TFLOPS, 4), "traffic": traffic},
     }
     if not args.no_secondary:
         line["secondary"] = secondary(rt, args.steps, args.warmup, args.extended)
