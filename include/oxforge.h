@@ -219,10 +219,11 @@ forge_status forge_fill(forge_runtime *rt, forge_stream *stream,
  * products, sums that are not finite, and sums to which what bf16's smallest
  * value cuts off operands under 2^-110 could matter are formed by the f32
  * matrix instructions (v_mfma_f32_16x16x4_f32).  Any M, N, K >= 0 (the reference
- * asserts multiples of 16).  Outputs whose tiles leave three quarters of the
- * CUs idle, with K >= 2048, are computed as K slices summed in slice order
- * (deterministic; tile, sum order and slices depend only on M, N and K, the
- * same for this call and forge_gemm_ex_f32). */
+ * asserts multiples of 16).  From K = 2048 on, outputs of few tiles are
+ * computed as K slices summed in slice order where a time model of the tiles
+ * finds that faster (deterministic; tile, sum order and slices depend only on
+ * M, N and K, above row pitches of 2^23 floats also on the orientation, and
+ * are the same for this call and forge_gemm_ex_f32). */
 forge_status forge_gemm_f32(forge_runtime *rt, forge_stream *stream,
                             forge_slice A, forge_slice B, forge_slice C,
                             size_t M, size_t N, size_t K);
