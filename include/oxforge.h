@@ -315,8 +315,9 @@ forge_status forge_gemm_sum_f32(forge_runtime *rt, forge_stream *stream, int tra
  * explicit plain tile instance: "<BM>x<BN>x<BK>_x" for the unguarded tiles of
  * one group of four waves (128x256x32, 128x128x32, 128x64x32, 64x128x32,
  * 64x64x32), "64x128x32_x8" and "64x64x32_x16" for two and four groups that
- * share out K, or "128x128x32_2x2_g", "64x64x16_2x2_g", "64x128x32_2x2_g8" and
- * "64x64x32_2x2_g16" for the guarded ones.
+ * share out K, "32x32x32_d" for the direct one, or "128x128x32_2x2_g",
+ * "64x64x16_2x2_g", "64x128x32_2x2_g8", "64x64x32_2x2_g16" and
+ * "32x32x32_2x2_gd" for guarded ones (row pitches to 2^23; 64x64x16_2x2_g any).
  * Unguarded tiles require M % BM == N % BN == K % BK == 0, 16-byte aligned
  * operands and K, N <= 2^21; anything else is FORGE_EINVAL.  A suffix
  * "@<n>" (1..16) lets a CU hold at most n of the launch's workgroups (the
