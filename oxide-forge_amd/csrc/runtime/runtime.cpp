@@ -845,7 +845,10 @@ double tile_time(const TileTimes& c, double cus, size_t M, size_t N, size_t coun
 // Tile choice by M, N and K alone, so that every entry point, epilogue,
 // orientation and batch forms a product of one shape in the same sum order
 // (the groups of a tile split K): for a batch, the best of the tiles with the
-// groups that one product takes.  Shapes the tile does not divide take its
+// groups that one product takes.  (Of direct products that is the direct tile
+// again, also over several rounds: three of 512 x 512 x 512 16.7 us, 11.3 on the
+// 64 x 64 tile, on which a single one takes 10.7 instead of 6.2.)  Shapes the
+// tile does not divide take its
 // guarded instance.  Groups of four waves pay from four slabs on (even one
 // slab each loads them all at once), the direct tile's at any K.
 const TileTimes& choose_shape(forge_runtime* rt, size_t M, size_t N, size_t K, size_t count = 1,
